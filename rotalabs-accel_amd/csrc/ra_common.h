@@ -44,6 +44,27 @@ __device__ __forceinline__ uint4 load_stream16(const void *p) {
   return make_uint4(v.x, v.y, v.z, v.w);
 }
 
+// 16-byte global load and 8- / 16-byte store at any byte address (gfx950
+// serves them unaligned; the compiler emits one dword-wide instruction), for
+// rows whose start or length is no multiple of 16 bytes.
+typedef u32x4_vec u32x4_any __attribute__((aligned(1)));
+typedef u32x2_t u32x2_any __attribute__((aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
+__device__ __forceinline__ uint4 load16_any(const void *p) {
+  const u32x4_vec v = *static_cast<const u32x4_any *>(p);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ uint4 load_stream16_any(const void *p) {  // non-temporal
+  const u32x4_vec v = __builtin_nontemporal_load(static_cast<const u32x4_any *>(p));
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ void store16_any(void *p, const uint4 &v) {
+  *static_cast<u32x4_any *>(p) = u32x4_vec{v.x, v.y, v.z, v.w};
+}
+__device__ __forceinline__ void store8_any(void *p, uint32_t lo, uint32_t hi) {
+  *static_cast<u32x2_any *>(p) = u32x2_t{lo, hi};
+}
+
 // One 32-bit (16-bit) word through the vector memory path (a buffer load)
 // although its address is wave-uniform. The decode kernels load their
 // epilogue operands (scale, bias) this way: as scalar loads they share the
