@@ -14,6 +14,38 @@ from oracle import fallback
 HALF = [torch.float16, torch.bfloat16]
 
 
+def test_fp32_quotient_without_a_division(tmp_path):
+    src = os.path.join(os.path.dirname(os.path.abspath(__file__)), "division_f32_check.c")
+    exe = str(tmp_path / "division_f32_check")
+    subprocess.run(["gcc", "-O2", "-ffp-contract=off", "-mfma", "-o", exe, src, "-lm"], check=True)
+    res = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    assert res.returncode == 0, res.stdout
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", HALF + [torch.float32])
+@pytest.mark.parametrize("n,k", [(5, 3), (5, 8), (7, 9), (3, 300), (6, 511), (9, 513), (5, 1025), (3, 2051),
+                                 (5, 4096), (2, 4099), (3, 8200), (2, 16384), (2, 16391)])
+def test_quantize_widths_bit_exact(gpu, dt, n, k):
+    """Codes and scales equal the CPU op sequence bit for bit: random rows, an
+    all-zero, a tiny-valued, a tie-valued and a NaN row."""
+    g = torch.Generator().manual_seed(n * k)
+    w = (torch.randn(n + 4, k, generator=g) * 0.02).to(dt)
+    w[n] = 0
+    w[n + 1] *= 1e-5 if dt == torch.float16 else 1e-33
+    w[n + 2] = ((torch.arange(k) % 254 - 127).float() + 0.5).clamp(-127, 127) / 8
+    w[n + 2, 0] = 127 / 8
+    w[n + 3, k // 2] = float("nan")
+    print(f"  quantize {dt} [{n + 4}, {k}]", flush=True)
+    # a view one row into a buffer of odd row length: rows at any address
+    buf = torch.empty(n + 5, k, dtype=dt, device=gpu)
+    buf[1:] = w.to(gpu)
+    q, s = ra.quantize_weight_per_channel(buf[1:])
+    q_c, s_c = ra.quantize_weight_per_channel(w)
+    assert torch.equal(q.cpu(), q_c)
+    torch.testing.assert_close(s.cpu(), s_c, rtol=0, atol=0, equal_nan=True)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", HALF + [torch.float32])
 @pytest.mark.parametrize("rows,hidden", [(1, 1), (3, 5), (7, 8), (5, 333), (9, 4104), (300, 2049)])
