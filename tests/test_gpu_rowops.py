@@ -72,3 +72,28 @@ def test_swiglu_tails(gpu, dt, rows, hidden, bias):
     # a relative error of g by at most 1 + |g|; then one rounding to dt
     unit = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -22}[dt]
     np.testing.assert_allclose(y.cpu().double().numpy(), ref, rtol=unit * 1.01 + 2.0 ** -19, atol=1e-6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", HALF)
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("rows,hidden", [(3, 7), (5, 8), (9, 9), (4, 2047), (3, 2056), (5, 4097), (2, 8199), (2, 16383)])
+def test_rmsnorm_odd_rows(gpu, dt, wide, rows, hidden):
+    """Ragged rows and fp32 weights: bit for bit the exactly rounded
+    restatement (its value before the weight, times the weight, for fp32)."""
+    g = torch.Generator().manual_seed(rows * hidden)
+    x = (torch.randn(rows, hidden, generator=g) * 2).to(dt)
+    r = (torch.randn(rows, hidden, generator=g) * 2).to(dt)
+    w = (1 + 0.01 * torch.randn(hidden, generator=g)).to(torch.float32 if wide else dt)
+    print(f"  rmsnorm {dt} [{rows}, {hidden}] wide={wide}", flush=True)
+    name = "f16" if dt == torch.float16 else "bf16"
+    for res in (None, r):
+        v = x if res is None else x + res
+        if res is None:
+            y = ra.rmsnorm(x.to(gpu), w.to(gpu), 1e-6).cpu()
+        else:
+            y = ra.rmsnorm_residual_fused(x.to(gpu), res.to(gpu), w.to(gpu), 1e-6).cpu()
+        one = np.ones(hidden, dtype=np.float32)
+        n = fallback.rmsnorm_exact_ref(v.float().numpy(), one, 1e-6, name)
+        ref = (torch.from_numpy(n) * w.float()).to(w.dtype)
+        assert y.dtype == w.dtype and torch.equal(y, ref)
