@@ -266,6 +266,15 @@ int ra_quantize_rows(const void *t, int64_t ldt, int t_dtype,
                      int8_t *q, int64_t ldq, void *scale, void *stream);
 
 /*
+ * The codec's way back (QuantizedTensor.dequantize, src/rotalabs_accel/
+ * speculative/kv_compression.py:80-84): out[r,c] = q[r,c] * scale[r] in fp32,
+ * rounded once to t_dtype. q: int8 [rows, cols]; scale: [rows] and out:
+ * [rows, cols] in t_dtype, all contiguous.
+ */
+int ra_dequantize_rows(const int8_t *q, const void *scale, int t_dtype,
+                       int64_t rows, int64_t cols, void *out, void *stream);
+
+/*
  * W8A8 route, step 1: per-row dynamic int8 quantisation of the activations
  * x[M,K] (fp16 or bf16), as _int8_gemm_cublas computes it
  * (src/rotalabs_accel/kernels/quantized_matmul.py:85-87), every op rounded to

@@ -558,6 +558,15 @@ int ra_quantize_rows(const void *t, int64_t ldt, int t_dtype, int64_t rows, int6
                                         static_cast<hipStream_t>(stream)));
 }
 
+int ra_dequantize_rows(const int8_t *q, const void *scale, int t_dtype, int64_t rows, int64_t cols, void *out,
+                       void *stream) {
+  if (rows < 0 || cols < 0 || rows > INT32_MAX || cols > INT32_MAX) return RA_ERR_ARG;
+  if (!valid_act(t_dtype)) return RA_ERR_DTYPE;
+  if (rows == 0 || cols == 0) return RA_OK;
+  if (!q || !scale || !out) return RA_ERR_ARG;
+  return to_status(dequantize_rows_launch(q, scale, t_dtype, rows, cols, out, static_cast<hipStream_t>(stream)));
+}
+
 int ra_quantize_act_rows(const void *x, int64_t ldx, int x_dtype, int64_t M, int64_t K, int8_t *q, int64_t ldq,
                          void *xs, float act_scale, void *stream) {
   if (M < 0 || K < 0 || M > INT32_MAX || K > INT32_MAX) return RA_ERR_ARG;

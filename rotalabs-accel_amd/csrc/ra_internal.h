@@ -136,6 +136,8 @@ hipError_t quantize_launch(const void *w, int64_t ldw, int w_dt, int64_t N, int6
                            int64_t ldq, float *scale, hipStream_t s);
 hipError_t quantize_rows_launch(const void *t, int64_t ldt, int t_dt, int64_t rows, int64_t cols, int bits,
                                 int8_t *q, int64_t ldq, void *scale, hipStream_t s);
+hipError_t dequantize_rows_launch(const int8_t *q, const void *scale, int t_dt, int64_t rows, int64_t cols, void *out,
+                                  hipStream_t s);
 
 // W8A8 (int8 activations x int8 weights on the int8 matrix cores).
 struct W8A8Args {

@@ -16,6 +16,8 @@ import torch
 
 from rotalabs_accel import _backend
 
+_KERNEL_DTYPES = (torch.float16, torch.bfloat16, torch.float32)
+
 
 class QuantizedTensor:
     """Quantized tensor for KV-cache compression (int8 storage for 8 and 4 bits)."""
@@ -29,7 +31,7 @@ class QuantizedTensor:
         if bits not in (8, 4):
             raise ValueError(f"Unsupported bits: {bits}")
         qmax = 2 ** (bits - 1) - 1
-        if per_channel and tensor.is_cuda and tensor.dtype in (torch.float16, torch.bfloat16, torch.float32) \
+        if per_channel and tensor.is_cuda and tensor.dtype in _KERNEL_DTYPES \
                 and tensor.dim() > 0:
             self.data, self.scale = self._quantize_rows_hip(tensor, bits)
             return
@@ -60,7 +62,22 @@ class QuantizedTensor:
         return q.view(tensor.shape), scale.view(tensor.shape[:-1] + (1,))
 
     def dequantize(self) -> torch.Tensor:
-        return self.data.to(self.dtype) * self.scale
+        q, s = self.data, self.scale
+        if isinstance(s, torch.Tensor) and q.is_cuda and q.dtype == torch.int8 and s.device == q.device \
+                and s.dtype == self.dtype and s.dtype in _KERNEL_DTYPES and q.dim() > 0 \
+                and s.shape == q.shape[:-1] + (1,) and q.is_contiguous() and s.is_contiguous() \
+                and not s.requires_grad and s.numel() < 1 << 31 and q.shape[-1] < 1 << 31:
+            return self._dequantize_rows_hip(q, s)
+        return q.to(self.dtype) * s
+
+    @staticmethod
+    def _dequantize_rows_hip(q: torch.Tensor, s: torch.Tensor) -> torch.Tensor:
+        lib = _backend.load()
+        out = torch.empty(q.shape, dtype=s.dtype, device=q.device)
+        with _backend.on_device(q.device):
+            _backend.check(lib.ra_dequantize_rows(q.data_ptr(), s.data_ptr(), _backend.dtype_code(s.dtype), s.numel(),
+                                                  q.shape[-1], out.data_ptr(), _backend.stream_handle(q.device)))
+        return out
 
     @property
     def memory_bytes(self) -> int:

@@ -75,6 +75,18 @@ def test_swiglu_tails(gpu, dt, rows, hidden, bias):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dt", HALF + [torch.float32])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 7), (1, 8), (5, 36), (131, 80), (1030, 128), (7, 1000), (2, 8200)])
+def test_kv_decode_bit_exact(gpu, dt, rows, cols):
+    from rotalabs_accel.speculative import QuantizedTensor
+    g = torch.Generator().manual_seed(rows + cols)
+    t = (torch.randn(rows, cols, generator=g) * 4).to(dt)
+    print(f"  kv decode {dt} [{rows}, {cols}]", flush=True)
+    qt = QuantizedTensor(t.to(gpu))
+    torch.testing.assert_close(qt.dequantize().cpu(), qt.data.cpu().to(dt) * qt.scale.cpu(), rtol=0, atol=0)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dt", HALF)
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("rows,hidden", [(3, 7), (5, 8), (9, 9), (4, 2047), (3, 2056), (5, 4097), (2, 8199), (2, 16383)])
