@@ -56,9 +56,11 @@ enum ra_variant {
   RA_VARIANT_ROWS = 5,    /* decode row GEMV, M <= 2, one weight row per wave */
   RA_VARIANT_BATCH = 6,   /* small batch, M <= 64, K % 128 == 0, MFMA + LDS */
   RA_VARIANT_SPLITK = 7,  /* small batch, M <= 64, K % 128 == 0, split K      */
-  RA_VARIANT_SPLITK_SPREAD = 8 /* the same with a row block's K splits run on
+  RA_VARIANT_SPLITK_SPREAD = 8, /* the same with a row block's K splits run on
                                   different XCDs (tests the exchange of the
                                   partial sums across XCDs)                  */
+  RA_VARIANT_STAGED = 9 /* register-staged MFMA GEMM: fp32 activations, rows of
+                           any alignment, K >= 16                            */
 };
 
 /* Version of this ABI (RA_ABI_VERSION of the built library). */

@@ -37,6 +37,7 @@ int g_w8a8_mode = 0;
 int g_gu_splitk = 0;
 int g_gu_rows = 0;
 int g_rows_lds = 0;
+int g_staged_cfg = 0;
 }
 #endif
 #ifdef RA_TRACE
@@ -275,7 +276,7 @@ int select_variant(const GemmArgs &a, bool have_ws) {
   if (gemv_supported(a)) return RA_VARIANT_GEMV;
   if (tiled_supported(a)) return RA_VARIANT_TILED;
   if (skinny_supported(a)) return RA_VARIANT_SKINNY;
-  return RA_VARIANT_GENERIC;
+  return staged_selected(a) ? RA_VARIANT_STAGED : RA_VARIANT_GENERIC;
 }
 
 // A caller workspace must start on an RA_WORKSPACE_ALIGN boundary (the
@@ -334,6 +335,7 @@ void ra_tune_tiled_split(int v) { ra::g_tiled_split = v; }
 void ra_tune_w8a8(int mode) { ra::g_w8a8_mode = mode; }
 void ra_tune_rows_lds(int v) { ra::g_rows_lds = v; }
 void ra_tune_gu_splitk(int v) { ra::g_gu_splitk = v; }
+void ra_tune_staged(int v) { ra::g_staged_cfg = v; }
 void ra_tune_gu_rows(int v) { ra::g_gu_rows = v; }
 #endif
 #ifdef RA_TRACE
@@ -406,6 +408,9 @@ int ra_w8a16_gemm_ex(const void *x, int64_t ldx, int x_dtype, const int8_t *w, i
     case RA_VARIANT_TILED:
       if (!tiled_supported(a) || K == 0) return RA_ERR_VARIANT;
       return to_status(tiled_launch_ws(a, have_ws ? workspace : nullptr, workspace_bytes, s));
+    case RA_VARIANT_STAGED:
+      if (!staged_supported(a)) return RA_ERR_VARIANT;
+      return to_status(staged_launch(a, s));
     case RA_VARIANT_GENERIC:
       return to_status(generic_launch(a, s));
     default:

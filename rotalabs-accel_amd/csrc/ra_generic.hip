@@ -1,7 +1,8 @@
 // Generic W8A16 kernels: any M, N, K, leading dimensions, alignment and
 // activation dtype (fp16, bf16, fp32). Plain VALU dot products, one wave per
-// output channel and four activation rows; used where the MFMA kernels'
-// alignment / K % 16 requirements do not hold and for fp32 activations.
+// output channel and four activation rows; used where neither the MFMA
+// kernels' alignment / K % 16 requirements hold nor the register-staged kernel
+// (ra_staged.hip) pays: tiny weights with a few rows, K < 16.
 // Same arithmetic contract as the fast kernels: exact int8, fp32 accumulation,
 // scale (and bias) applied to the fp32 sum, one rounding to the output dtype.
 #include "ra_common.h"

@@ -59,6 +59,12 @@ hipError_t tiled_launch_ws(const GemmArgs &a, void *ws, size_t ws_bytes, hipStre
 // Generic kernel: any shape, alignment and activation dtype.
 hipError_t generic_launch(const GemmArgs &a, hipStream_t s);
 
+// Register-staged MFMA kernel: fp32 activations (exact bf16 split), rows at
+// any alignment and any K >= 16.
+bool staged_supported(const GemmArgs &a);
+bool staged_selected(const GemmArgs &a);  // ... and ahead of the VALU kernel
+hipError_t staged_launch(const GemmArgs &a, hipStream_t s);
+
 // Fused gate/up + SwiGLU.
 struct GateUpArgs {
   const void *x;

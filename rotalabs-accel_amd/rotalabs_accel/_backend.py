@@ -30,7 +30,7 @@ WORKSPACE_COUNTER_BYTES = 16384
 F16, BF16, F32 = 0, 1, 2
 # enum ra_variant
 (VARIANT_AUTO, VARIANT_SKINNY, VARIANT_TILED, VARIANT_GENERIC, VARIANT_GEMV, VARIANT_ROWS, VARIANT_BATCH,
- VARIANT_SPLITK, VARIANT_SPLITK_SPREAD) = range(9)
+ VARIANT_SPLITK, VARIANT_SPLITK_SPREAD, VARIANT_STAGED) = range(10)
 
 _DTYPE_CODE = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}
 
