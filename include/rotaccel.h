@@ -54,8 +54,8 @@ enum ra_variant {
   RA_VARIANT_GENERIC = 3, /* any shape / alignment / dtype, VALU, slow        */
   RA_VARIANT_GEMV = 4,    /* decode GEMV, M <= 4, x staged in LDS             */
   RA_VARIANT_ROWS = 5,    /* decode row GEMV, M <= 2, one weight row per wave */
-  RA_VARIANT_BATCH = 6,   /* small batch, M <= 64, K % 128 == 0, MFMA + LDS */
-  RA_VARIANT_SPLITK = 7,  /* small batch, M <= 64, K % 128 == 0, split K      */
+  RA_VARIANT_BATCH = 6,   /* small batch, M <= 64, K % 32 == 0, MFMA + LDS  */
+  RA_VARIANT_SPLITK = 7,  /* small batch, M <= 64, K % 32 == 0, split K       */
   RA_VARIANT_SPLITK_SPREAD = 8, /* the same with a row block's K splits run on
                                   different XCDs (tests the exchange of the
                                   partial sums across XCDs)                  */

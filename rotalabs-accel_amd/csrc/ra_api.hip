@@ -78,7 +78,7 @@ constexpr int64_t kSplitkMinK = 16384;
 int one_row_short_k(const GemmArgs &a) {
   if (a.M != 1 || a.K > 2048 || a.N < 4096) return 0;
   if (a.K <= 1536 && a.N >= 16384 && skinny_supported(a)) return RA_VARIANT_SKINNY;
-  return batch_supported(a) ? RA_VARIANT_BATCH : 0;
+  return a.K % 128 == 0 && batch_supported(a) ? RA_VARIANT_BATCH : 0;
 }
 
 // M = 33..56 at short K over at most ~12K weight rows: the small-batch
@@ -125,6 +125,8 @@ bool short_k_batch(const GemmArgs &a) {
 //    +25 %, K=4096 N=28672 +23 %; level at K=1024 N=28672), from K = 4096
 //    over 6144+ rows (M=40 K=5120 N=11008 +19 %, K=4096 N=6144 +15 %; level
 //    at K=4096 N=8192-16384), at K = 3072 over at most 2048 rows (M=40 +9 %);
+//    the tiles are ahead over 8192+ rows below K = 5120 where K % 128 != 0
+//    adds a tail stage here (K=4160 N=8192 18.0 against 19.3);
 //    the tiles and the small-batch kernel stay ahead at K <= 2048 below 28672
 //    rows (M=48 K=2048 N=11008 24 % behind) and at K = 3072 over 4096-16384.
 //  * M = 49..64 (four 16-row tiles): below 8192 rows from K = 4096 and
@@ -169,7 +171,8 @@ bool splitk_wanted(const GemmArgs &a) {
   if (a.N >= 28672) return true;
   if (a.M == 33) {
     if ((a.K >= 4096 && a.N >= 11008) || (a.K >= 5120 && a.N >= 6144)) return true;
-  } else if ((a.K >= 4096 && a.N >= 6144) || (a.K >= 3072 && a.N <= 2048)) {
+  } else if ((a.K >= 4096 && a.N >= 6144 && (a.K % 128 == 0 || a.K >= 5120 || a.N < 8192)) ||
+             (a.K >= 3072 && a.N <= 2048)) {
     return true;
   }
   if (a.N <= 4096) return a.K >= 4096;
@@ -248,6 +251,8 @@ int select_variant(const GemmArgs &a, bool have_ws) {
   // (8.5 vs 9.8 at K=4096 N=11008, 37.3 vs 39.0 at K=28672).
   const bool two_rows_few =
       a.M == 2 && (a.N <= 1024 || (a.N <= 2048 && a.K >= 8192 && a.K <= 16384));
+  // (K % 128 != 0: two rows take the skinny kernel, as 3..16 rows do below;
+  // K=4128 N=8192 16.5 -> 11.3 us)
   if (gemv_rows_supported(a) && (a.M == 1 || two_rows_few || !batch_supported(a))) {
     const int v = one_row_short_k(a);
     return v ? v : RA_VARIANT_ROWS;
@@ -269,9 +274,12 @@ int select_variant(const GemmArgs &a, bool have_ws) {
     if (p.ok && (p.S == 1 || have_ws)) return RA_VARIANT_SPLITK;
   }
   // M = 3..64: the small-batch kernel (line-wide weight loads, activations
-  // read once per 48 rows) where K % 128 == 0, else the split-K MFMA kernel;
-  // both measured faster than the LDS GEMV, which stays as a fallback.
-  if (a.M <= kSkinnyMaxM && batch_supported(a)) return RA_VARIANT_BATCH;
+  // read once per 48 rows) where K % 128 == 0, or K % 32 == 0 from 17 rows
+  // (a tail stage; bf16, us, skinny kernel -> small batch, K=4160 / 4128
+  // N=8192: M=17 17.3 / 17.2 -> 14.0 / 15.6, M=32 23.0 / 22.3 -> 17.5 / 17.9;
+  // M=8 11.9 / 12.5 against 12.4 / 14.3), else the split-K MFMA kernel; both
+  // measured faster than the LDS GEMV, which stays as a fallback.
+  if (a.M <= kSkinnyMaxM && batch_supported(a) && (a.K % 128 == 0 || a.M > 16)) return RA_VARIANT_BATCH;
   if (a.M <= kSkinnyMaxM && skinny_supported(a)) return RA_VARIANT_SKINNY;
   if (gemv_supported(a)) return RA_VARIANT_GEMV;
   if (tiled_supported(a)) return RA_VARIANT_TILED;

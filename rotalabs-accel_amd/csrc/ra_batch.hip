@@ -88,7 +88,7 @@ __global__ __launch_bounds__(NW * 64) void batch_kernel(const uint16_t *__restri
 
   const int kb = wid * kslice;
   const int ke = min(K, kb + kslice);
-  const int nst = ke > kb ? (ke - kb) / KS : 0;
+  const int nst = ke > kb ? (ke - kb + KS - 1) / KS : 0;
 
   f32x4 acc[NTW][MT];
 #pragma unroll
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(NW * 64) void batch_kernel(const uint16_t *__restri
   uint4 xf[D][4][MT];
 #define RA_LOAD_STAGE(st_, SLOT_)                                                                   \
   {                                                                                                 \
-    const int k_ = kb + KS * (st_);                                                                 \
+    const int k_ = min(kb + KS * (st_), K - KS); /* K % 128 != 0: the last stage ends at K */       \
     const int slot_ = (SLOT_);                                                                      \
     _Pragma("unroll") for (int j_ = 0; j_ < WL; ++j_) wreg[slot_][j_] =                             \
         load_stream16(wsrc[j_] + k_);                                                               \
@@ -124,6 +124,12 @@ __global__ __launch_bounds__(NW * 64) void batch_kernel(const uint16_t *__restri
   {                                                                                                 \
     _Pragma("unroll") for (int j = 0; j < WL; ++j)                                                  \
         store16(slot + wdst[j], wreg[DP_][j]);                                                     \
+    const int skip_ = GU ? 0 : kb + KS * (st_) + KS - K;                                            \
+    if (!GU && skip_ > 0) { /* activations of the k's that the stage before covers */               \
+      _Pragma("unroll") for (int s = 0; s < 4; ++s)                                                 \
+        if (32 * s + 8 * g < skip_)                                                                 \
+          _Pragma("unroll") for (int mt = 0; mt < MT; ++mt) xf[DP_][s][mt] = make_uint4(0, 0, 0, 0); \
+    }                                                                                               \
     _Pragma("unroll") for (int s = 0; s < 4; ++s) {                                                 \
       _Pragma("unroll") for (int t = 0; t < NTW; ++t) {                                             \
         const int row = 16 * t + r;                                                                 \
@@ -542,19 +548,23 @@ __global__ __launch_bounds__(64 * gux::kWaves) void gateup_xlds_kernel(
 // ----------------------------------------------------------------------------
 // Host side.
 // ----------------------------------------------------------------------------
+// kstep: K's granularity, 128 for the gate/up form (whose kernels have no tail
+// stage), 32 for the GEMM.
 static bool batch_shape_ok(int x_dt, const void *x, int64_t ldx, const int8_t *w, int64_t ldw, int64_t M,
-                           int64_t N, int64_t K) {
+                           int64_t N, int64_t K, int kstep) {
   if (x_dt != RA_F16 && x_dt != RA_BF16) return false;
   if (M < 1 || M > batch::kMaxM || N > ((int64_t)1 << 30) || K > ((int64_t)1 << 30)) return false;
-  if (K < batch::KS || K % batch::KS != 0) return false;
+  if (K < batch::KS || K % kstep != 0) return false;
   if ((reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(w) & 15)) return false;
   return (ldx % 8) == 0 && (ldw % 16) == 0;
 }
 
-bool batch_supported(const GemmArgs &a) { return batch_shape_ok(a.x_dt, a.x, a.ldx, a.w, a.ldw, a.M, a.N, a.K); }
+bool batch_supported(const GemmArgs &a) {
+  return batch_shape_ok(a.x_dt, a.x, a.ldx, a.w, a.ldw, a.M, a.N, a.K, 32);
+}
 
 bool gateup_batch_supported(const GateUpArgs &a) {
-  return batch_shape_ok(a.x_dt, a.x, a.ldx, a.w, a.ldw, a.M, a.I, a.K);
+  return batch_shape_ok(a.x_dt, a.x, a.ldx, a.w, a.ldw, a.M, a.I, a.K, batch::KS);
 }
 
 template <int DT, int MT, int RT, int NW, bool GU>

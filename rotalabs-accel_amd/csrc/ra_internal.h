@@ -37,7 +37,7 @@ hipError_t skinny_launch(const GemmArgs &a, const SkinnyCfg &c, hipStream_t s);
 // Tiled (LDS-staged MFMA) kernel for large M.
 bool tiled_supported(const GemmArgs &a);
 // Whether the automatic choice runs the tiled kernel with its 64 x 64 tile
-// (M = 33..64, at least 8192 weight rows, K % 64 == 0).
+// (M = 33..64, at least 8192 weight rows, K >= 64).
 bool tiled_small_selected(const GemmArgs &a);
 hipError_t tiled_launch(const GemmArgs &a, hipStream_t s);
 // M = 33..64 (where tiled_small_selected): the small tile with K split over
@@ -89,14 +89,15 @@ hipError_t gemv_rows_launch(const GemmArgs &a, hipStream_t s);
 bool gateup_gemv_rows_supported(const GateUpArgs &a);
 hipError_t gateup_gemv_rows_launch(const GateUpArgs &a, hipStream_t s);
 
-// Small-batch MFMA GEMM (M <= 64, K % 128 == 0): line-wide weight loads
+// Small-batch MFMA GEMM (M <= 64, K % 32 == 0 from 128; the gate/up form
+// K % 128 == 0): line-wide weight loads
 // transposed through LDS, split-K across the workgroup's waves.
 bool batch_supported(const GemmArgs &a);
 hipError_t batch_launch(const GemmArgs &a, hipStream_t s);
 bool gateup_batch_supported(const GateUpArgs &a);
 hipError_t gateup_batch_launch(const GateUpArgs &a, hipStream_t s);
 
-// Small-batch GEMM with split K (M <= 64, K % 128 == 0): weights and
+// Small-batch GEMM with split K (M <= 64, K as above): weights and
 // activations staged by direct-to-LDS copies; S > 1 needs a workspace of
 // ws_bytes (a zeroed counter block of cnt_bytes, then the partial sums).
 // Bytes of the counter block at the start of every split-K workspace (must

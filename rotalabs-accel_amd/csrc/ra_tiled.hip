@@ -228,7 +228,7 @@ __global__ __launch_bounds__(256, 2) void tiled_kernel(const uint16_t *__restric
 }
 
 // ---------------------------------------------------------------------------
-// Multi-stage variant for K % 64 == 0: the global -> LDS copies are gfx950
+// Multi-stage variant for K >= 64 (K % 16 == 0 as everywhere here): the global -> LDS copies are gfx950
 // direct-to-LDS loads (global_load_lds_dwordx4: each lane's 16 bytes land at
 // M0 + 16 * lane, no VGPR round trip), S K-tiles deep, so S-1 tiles are in
 // flight while one is multiplied. The XOR swizzles are applied on the global
@@ -242,6 +242,14 @@ __global__ __launch_bounds__(256, 2) void tiled_kernel(const uint16_t *__restric
 // 16q + 15, q = 2p + g) once per pair p of sub-steps; sub-step s = 2p + h
 // uses its 8-byte half h, and A supplies the same k's (8-half chunk
 // 4p + 2g + h), so the B read is shared by two MFMA sub-steps.
+// K % 64 != 0, pad k's short of whole tiles: tile 1 starts at 64 - pad, and so
+// on to a last tile that ends at K (no copy leaves the rows, and only tile 0
+// is off the common origin); the activations in tile 0 of the k's that tile 1
+// holds too are cleared in LDS before the first read, so the K loop is the
+// same code. (Moving the last tile instead, or masking fragments, slowed the
+// whole multiples: M=2048 K=4096 N=8192 103 -> 126 us.) The register-staged
+// kernel above ran these with 256-row tiles, whatever M, and no split (bf16,
+// us, N=4096 K=11040: M=100 224 -> 33, M=2048 247 -> 157).
 // ---------------------------------------------------------------------------
 // Largest byte offset the 32-bit per-lane copy offsets may reach. The copy
 // bases are moved down by DMA_BIAS so that offsets minus the instruction
@@ -394,8 +402,10 @@ __global__ __launch_bounds__(256, 1) void tiled_dma_kernel(const uint16_t *__res
     }
     b_voff[i] = (uint32_t)((int64_t)wr * ldw + c * 16) + (uint32_t)(DMA_BIAS - (i % 4) * 1024);
   }
-  const char *const xb = reinterpret_cast<const char *>(x) - DMA_BIAS;
-  const char *const wb = reinterpret_cast<const char *>(w) - DMA_BIAS;
+  const int KTA = (K + BK - 1) / BK;  // K tiles in all
+  const int pad = KTA * BK - K;       // k's that tiles 0 and 1 share
+  const char *const xb = reinterpret_cast<const char *>(x) - DMA_BIAS - 2 * pad;
+  const char *const wb = reinterpret_cast<const char *>(w) - DMA_BIAS - pad;
   const uint32_t lds0 = lds_offset(lds);
   const uint32_t a_dst = lds0 + (uint32_t)(A_COPIES * wid) * 1024;
   const uint32_t b_dst = lds0 + A_BYTES + (uint32_t)(B_COPIES * wid) * 1024;
@@ -409,6 +419,11 @@ __global__ __launch_bounds__(256, 1) void tiled_dma_kernel(const uint16_t *__res
 #define RA_ISSUE_PART(kt_, st_, LO_, HI_)                                                   \
   {                                                                                         \
     const int ko_ = uniform_if<SPLIT && (BMB > 1)>((kt0 + (kt_)) * BK);                     \
+    RA_ISSUE_AT(ko_, st_, LO_, HI_);                                                        \
+  }
+// ... of the K tile at element ko_ of the shifted rows.
+#define RA_ISSUE_AT(ko_, st_, LO_, HI_)                                                     \
+  {                                                                                         \
     const char *sa_ = xb + (int64_t)ko_ * 2;                                                \
     const char *sb_ = wb + (int64_t)ko_;                                                    \
     const uint32_t so_ = (uint32_t)(st_) * STAGE;                                           \
@@ -541,12 +556,23 @@ constexpr int P1 = (COPIES + 2) / 3, P2 = (2 * COPIES + 2) / 3;
   });                                                                                               \
   __builtin_amdgcn_sched_barrier(0);
 
-  const int KT = SPLIT ? min(K / BK - kt0, ksplit) : K / BK;  // K tiles of this workgroup (>= 1)
+  const int KT = SPLIT ? min(KTA - kt0, ksplit) : KTA;  // K tiles of this workgroup (>= 1)
+  const bool short0 = pad > 0 && kt0 == 0;              // this workgroup's tile 0 overlaps tile 1
+  const int ko0 = uniform_if<SPLIT && (BMB > 1)>(short0 ? pad : kt0 * BK);
+  RA_ISSUE_AT(ko0, 0, 0, COPIES);
 #pragma unroll
-  for (int s = 0; s < S; ++s)
+  for (int s = 1; s < S; ++s)
     if (s < KT) RA_ISSUE(s, s);
   wait_tiles<COPIES, S - 1>(min(KT, S) - 1);
   asm volatile("s_barrier" ::: "memory");
+  if (short0) {
+    const int c0 = (BK - pad) / 8, nc = 8 - c0;
+    for (int i = tid; i < BM * nc; i += 256) {
+      const int row = i / nc, c = c0 + i - row * nc;
+      store16(lds + row * 128 + ((c ^ ((row >> 1) & 7)) << 4), make_uint4(0, 0, 0, 0));
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
 #ifdef RA_TRACE
   tr_ready = __builtin_amdgcn_s_memrealtime();
 #endif
@@ -603,6 +629,7 @@ constexpr int P1 = (COPIES + 2) / 3, P2 = (2 * COPIES + 2) / 3;
 #undef RA_READ_A
 #undef RA_ISSUE
 #undef RA_ISSUE_PART
+#undef RA_ISSUE_AT
 
 #ifdef RA_TRACE
   tr_kend = __builtin_amdgcn_s_memrealtime();
@@ -780,8 +807,8 @@ static bool dma_span_ok(bool gu, int64_t ldx, int64_t ldw, int64_t N, int64_t K,
 }
 
 bool tiled_small_selected(const GemmArgs &a) {
-  return a.M >= kSmallTileMinM && a.M <= kSmallTileMaxM && a.N >= kSmallTileMinN && a.K > 0 &&
-         a.K % tiled::BK == 0 && tiled_supported(a) && dma_span_ok(false, a.ldx, a.ldw, a.N, a.K, 256);
+  return a.M >= kSmallTileMinM && a.M <= kSmallTileMaxM && a.N >= kSmallTileMinN && a.K >= tiled::BK &&
+         tiled_supported(a) && dma_span_ok(false, a.ldx, a.ldw, a.N, a.K, 256);
 }
 
 // M = 65..1024: the large tiles leave most CUs idle where N is small (M=128
@@ -791,7 +818,7 @@ bool tiled_small_selected(const GemmArgs &a) {
 static bool tiled_split_eligible(const GemmArgs &a) {
   if (tiled_small_selected(a)) return true;
   // One launch covers all rows of x (its copies' 31-bit offsets).
-  return a.M > kSmallTileMaxM && a.M <= kSplitTileMaxM && a.K > 0 && a.K % tiled::BK == 0 &&
+  return a.M > kSmallTileMaxM && a.M <= kSplitTileMaxM && a.K >= tiled::BK &&
          tiled_supported(a) && dma_span_ok(false, a.ldx, a.ldw, a.N, a.K, (int)std::max<int64_t>(a.M, 256));
 }
 
@@ -854,7 +881,7 @@ TiledSplitPlan tiled_split_plan(const GemmArgs &a) {
     const bool mid = a.M > 4 * kSmallTileMaxM && a.M <= 6 * kSmallTileMaxM;
     if (mid ? (lt >= cus || a.N > 16384) : 2 * lt >= cus) return best;
   }
-  const int64_t KT = a.K / tiled::BK;
+  const int64_t KT = (a.K + tiled::BK - 1) / tiled::BK;
   const int64_t tiles_m = (a.M + 63) / 64;
   auto cost = [&](int bmb, int bnb, int nsplit, int64_t ksplit) {
     const int64_t tiles = (tiles_m + bmb - 1) / bmb * ((a.N + 64 * bnb - 1) / (64 * bnb));
@@ -1043,10 +1070,10 @@ static hipError_t launch(const void *x, int64_t ldx, int x_dt, const int8_t *w, 
 #ifdef RA_TUNING
   extern int g_tiled_mode;  // 0 auto, 1 register-staged kernel, 2 direct-to-LDS auto, 3.. forced shapes (5 = 256x256 1x4, 7 = 256x256 2x2)
   forced = g_tiled_mode;
-  const bool use_dma = (g_tiled_mode >= 2 || (g_tiled_mode == 0 && K % tiled::BK == 0)) &&
+  const bool use_dma = (g_tiled_mode >= 2 || (g_tiled_mode == 0 && K >= tiled::BK)) &&
                        dma_span_ok(GU, ldx, ldw, N, K, 256);
 #else
-  const bool use_dma = K % tiled::BK == 0 && dma_span_ok(GU, ldx, ldw, N, K, 256);
+  const bool use_dma = K >= tiled::BK && dma_span_ok(GU, ldx, ldw, N, K, 256);
 #endif
   if (use_dma) {
     if (x_dt == RA_F16)
