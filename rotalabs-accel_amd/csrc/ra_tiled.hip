@@ -278,6 +278,7 @@ struct DmaTile {
   // pipeline depth: up to 4 stages, up to SMAX for small tiles
   static constexpr int SMAX = STAGE <= 24 * 1024 ? SMAX_SMALL : 4;
   static constexpr int S = (160 * 1024) / STAGE < SMAX ? (160 * 1024) / STAGE : SMAX;
+  static constexpr int PER_CU = S * STAGE <= 80 * 1024 && SMAX_SMALL < 6 ? 2 : 1;  // workgroups per CU aimed at
   static_assert(A_BYTES % 4096 == 0 && B_BYTES % 4096 == 0, "copies must split evenly over 4 waves");
   static_assert(S >= 2 && S <= 13, "2 to 13 stages");
   static_assert((S - 1) * COPIES <= 63, "vmcnt is a 6-bit counter");
@@ -318,7 +319,7 @@ constexpr int kMaxTileSplits = 4;  // K splits per tile of the SPLIT form
 constexpr int kMaxTileBmb = 2;     // 32x32 row blocks per wave of the SPLIT form (tiles of 64 or 128 rows)
 
 template <int DT, bool GU, int BMB, int BNB, int WR, int SM = 4, bool SPLIT = false>
-__global__ __launch_bounds__(256, 1) void tiled_dma_kernel(const uint16_t *__restrict__ x, int64_t ldx,
+__global__ __launch_bounds__(256, (DmaTile<BMB, BNB, WR, SM>::PER_CU)) void tiled_dma_kernel(const uint16_t *__restrict__ x, int64_t ldx,
                                                            const int8_t *__restrict__ w, int64_t ldw,
                                                            const float *__restrict__ scale,
                                                            const void *__restrict__ bias, int bias_dt,
@@ -1005,6 +1006,23 @@ static DmaShape pick_dma_shape(int64_t M, int64_t N, bool gu, int cus) {
   return best;
 }
 
+// Small grids: tiles of 64 x 128 (four stages) or 128 x 128 (three), two
+// workgroups per CU, where they fill at most one round of the CUs, one each.
+// A K tile then takes about 0.42 / 0.47 us, against 0.65-0.8 with 256 x 128
+// on fewer CUs. Gate/up, bf16, us, large tiles -> these: M=100 K=2048 I=5504
+// 32.8 -> 20.8, M=128 K=8192 I=2752 86.9 -> 54.0, M=400 88.0 -> 64.0; M=128
+// K=4096 I=11008 56.1 -> 38.1; M=200 K=2048 I=5504 37.1 -> 25.9 (64-row tiles,
+// past one round: 27.8). GEMM (beyond the split plans): M=512 K=N=8192 81.2
+// -> 70.0. Past one round they fall behind (gate/up M=200 K=4096 I=11008 60.5
+// against 57.0, M=300 88.7 against 80.5), but for the gate/up product up to
+// 128 rows, where any taller tile is mostly padding (M=100 K=8192 I=28672
+// 163.3 -> 146.0). Returns 64 or 128 (rows), 0: the large tiles.
+static int small_grid_rows(int64_t M, int64_t N, bool gu, int cus) {
+  const int64_t cols = gu ? (N + 63) / 64 : (N + 127) / 128;
+  if ((M + 63) / 64 * cols <= cus) return 64;
+  return (M + 127) / 128 * cols <= cus || (gu && M <= 128) ? 128 : 0;
+}
+
 static int64_t large_tile_count(int64_t M, int64_t N, int cus) {
   const DmaShape c = pick_dma_shape(M, N, false, cus);
   return ((M + c.bm() - 1) / c.bm()) * ((N + c.bn() - 1) / c.bn());
@@ -1034,8 +1052,6 @@ static void launch_dma_auto(const void *x, int64_t ldx, const int8_t *w, int64_t
     if (forced == 8) return launch_dma<DT, GU, 6, 2, 1>(x, ldx, w, ldw, scale, bias, bias_dt, y, ldy, M, N, K, s);
     if (forced == 9) return launch_dma<DT, GU, 7, 2, 1>(x, ldx, w, ldw, scale, bias, bias_dt, y, ldy, M, N, K, s);
   }
-#else
-  (void)forced;
 #endif
   // Up to 64 rows: 64 x 64 tiles (2 x 2 waves of one 32 x 32 block each),
   // six K tiles of copies in flight.
@@ -1052,6 +1068,9 @@ static void launch_dma_auto(const void *x, int64_t ldx, const int8_t *w, int64_t
     if (M <= kSmallTileMaxM)
       return launch_dma<DT, GU, 1, 1, 2, 6>(x, ldx, w, ldw, scale, bias, bias_dt, y, ldy, M, N, K, s);
   }
+  const int rows = forced ? 0 : small_grid_rows(M, N, GU, device_cus());
+  if (rows == 64) return launch_dma<DT, GU, 1, 2, 2, 4>(x, ldx, w, ldw, scale, bias, bias_dt, y, ldy, M, N, K, s);
+  if (rows == 128) return launch_dma<DT, GU, 2, 2, 2, 3>(x, ldx, w, ldw, scale, bias, bias_dt, y, ldy, M, N, K, s);
   if (c.wr == 1) return launch_dma<DT, GU, 8, 2, 1>(x, ldx, w, ldw, scale, bias, bias_dt, y, ldy, M, N, K, s);
   if (c.bmb == 3 && c.bnb == 4)
     return launch_dma<DT, GU, 3, 4, 2>(x, ldx, w, ldw, scale, bias, bias_dt, y, ldy, M, N, K, s);

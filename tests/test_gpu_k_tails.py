@@ -36,11 +36,13 @@ def test_small_batch_k_tails(gpu, dt, variant, M, K, N):
         assert torch.equal(gm._int8_gemm_hip(x, q, s, None, variant=variant).double(), exact)
 
 
-# Tiles: 64 rows (33..64), split plans (65..384), the large tiles; tails of
-# 16, 32 and 48 k, alone (K < 128) and after full tiles.
+# Tiles: 64 rows (33..64), split plans (65..384), two workgroups per CU (64 and
+# 128 rows), the large tiles (the last three); tails of 16, 32 and 48 k, alone
+# (K < 128) and after full tiles.
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,K,N", [(33, 80, 100), (64, 2096, 8200), (64, 112, 70), (65, 11056, 300), (200, 1072, 1030),
-                                   (300, 96, 333), (700, 368, 600), (2000, 304, 520), (1100, 144, 2100)])
+                                   (300, 96, 333), (700, 368, 600), (2000, 304, 520), (1100, 144, 2100),
+                                   (2100, 144, 4200), (1300, 80, 6000), (520, 112, 9000)])
 def test_tiled_k_tails(gpu, dt, M, K, N):
     x, q, s, exact = _case(M, K, N, dt, gpu)
     print(f"  k tail tiles {dt} M={M} K={K} N={N}", flush=True)
@@ -48,9 +50,11 @@ def test_tiled_k_tails(gpu, dt, M, K, N):
 
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("M,K,inter", [(70, 80, 100), (300, 1072, 520), (600, 368, 1000)])
+@pytest.mark.parametrize("M,K,inter", [(70, 80, 100), (300, 1072, 520), (600, 368, 1000), (128, 64, 17000),
+                                       (500, 128, 2050), (600, 368, 5000)])
 def test_gateup_tiled_k_tails(gpu, dt, M, K, inter):
-    """The gate/up tiles: the same sums as the GEMM's, one SwiGLU on top."""
+    """The gate/up tiles (64 and 128 rows, two workgroups per CU, and the large
+    ones): the same sums as the GEMM's, one SwiGLU on top."""
     from rotalabs_accel.kernels.mlp import int8_gateup_swiglu
     x, q, s, exact = _case(M, K, 2 * inter, dt, gpu)
     print(f"  k tail gate/up {dt} M={M} K={K} I={inter}", flush=True)
