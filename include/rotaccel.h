@@ -121,6 +121,12 @@ int ra_w8a16_gemm_ws(const void *x, int64_t ldx, int x_dtype,
 /* Workspace bytes ra_w8a16_gemm_ws may use for this problem (0: none). */
 size_t ra_w8a16_gemm_workspace_size(int64_t M, int64_t N, int64_t K, int x_dtype);
 
+/* Workspace bytes the automatic choice of ra_w8a16_gemm_ws makes use of for
+ * this problem with contiguous, 16-byte aligned operands: at most
+ * ra_w8a16_gemm_workspace_size, and 0 where the chosen kernel takes none. A
+ * call with this much runs as one with more. */
+size_t ra_w8a16_gemm_auto_workspace(int64_t M, int64_t N, int64_t K, int x_dtype);
+
 /*
  * ra_w8a16_gemm_ws without a caller workspace and without any allocation:
  * the split-K kernel's workspace is a fixed 16 MiB device array of the

@@ -380,6 +380,14 @@ size_t ra_w8a16_gemm_workspace_size(int64_t M, int64_t N, int64_t K, int x_dtype
   return sk > tiled ? sk : tiled;
 }
 
+size_t ra_w8a16_gemm_auto_workspace(int64_t M, int64_t N, int64_t K, int x_dtype) {
+  if (x_dtype != RA_F16 && x_dtype != RA_BF16) return 0;
+  if (M < 2 || M > kSplitTileMaxM || N < 1 || K < 1) return 0;
+  const GemmArgs a{reinterpret_cast<const void *>(256), K, x_dtype, reinterpret_cast<const int8_t *>(256),
+                   K, nullptr, nullptr, RA_F32, nullptr, N, M, N, K};
+  return auto_workspace_bytes(a);
+}
+
 int ra_w8a16_gemm_ex(const void *x, int64_t ldx, int x_dtype, const int8_t *w, int64_t ldw,
                      const float *scale, const void *bias, int bias_dtype, void *y, int64_t ldy, int64_t M,
                      int64_t N, int64_t K, int variant, void *workspace, size_t workspace_bytes, void *stream) {

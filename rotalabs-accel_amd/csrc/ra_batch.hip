@@ -628,14 +628,6 @@ static void batch_dispatch_rt(const void *x, int64_t ldx, const int8_t *w, int64
     batch_dispatch_mt<DT, RT, 4, GU>(x, ldx, w, ldw, scale, bias, bias_dt, y, ldy, M, N, K, s);
 }
 
-static int device_cus() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    return 256;
-  return cus;
-}
-
 // Weight tiles per workgroup. Each workgroup streams its 16*RT rows (times 2
 // with the gate/up pair) and reads the whole activation block once, so the
 // cost per CU is the rows of its busiest share plus the activation bytes of

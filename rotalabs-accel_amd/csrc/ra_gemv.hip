@@ -210,13 +210,6 @@ bool gateup_gemv_supported(const GateUpArgs &a) {
   return gemv_ok(a.x_dt, a.x, a.ldx, a.w, a.ldw, a.M, a.I, a.K, true);
 }
 
-static int device_cus() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) return 256;
-  return cus;
-}
-
 // Workgroups of this kernel that fit on one CU at once (registers, LDS, waves).
 template <typename Kern>
 static int resident_per_cu(Kern kern, int threads, size_t lds) {

@@ -11,6 +11,18 @@
 
 namespace ra {
 
+// CUs of the current device, asked for once per thread and device.
+inline int device_cus() {
+  thread_local int known = -1, cus = 256;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 256;
+  if (dev == known) return cus;
+  int n = 0;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 256;
+  known = dev;
+  return cus = n;
+}
+
 struct GemmArgs {
   const void *x;
   int64_t ldx;

@@ -481,14 +481,6 @@ bool x1_wanted(int64_t M, int64_t K, bool gu) {
   return M == 33 || (M == 17 && (gu || K >= 16384));
 }
 
-int device_cus() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    return 256;
-  return cus;
-}
-
 }  // namespace
 
 // Plan: waves per workgroup NW, tiles per wave TW and splits S minimising a
@@ -515,7 +507,7 @@ int device_cus() {
 // Splits whose partial sums exceed kSplitkMaxWorkspace are not considered
 // (at M=32 K=28672 N=32768 a 5-way split of 192-row blocks, 21 MB of partial
 // sums, measured 196.7 us against 171.7 unsplit).
-SplitkPlan splitk_plan(int64_t M, int64_t N, int64_t K, bool gu, bool allow_split) {
+static SplitkPlan make_plan(int64_t M, int64_t N, int64_t K, bool gu, bool allow_split, int cus) {
   SplitkPlan best{};
   best.ok = false;
   if (M < 1 || M > sk::kMaxM || K < sk::KS || K % (gu ? sk::KS : 32) != 0 || N < 1) return best;
@@ -524,7 +516,6 @@ SplitkPlan splitk_plan(int64_t M, int64_t N, int64_t K, bool gu, bool allow_spli
     mt = (int)(M / 16);
     x1 = 1;
   }
-  const int cus = device_cus();
   const int64_t xcd_cus = std::max(cus / 8, 1);
   const int64_t stages = (K + sk::KS - 1) / sk::KS;
   constexpr int kCuLds = 160 * 1024;
@@ -584,6 +575,29 @@ SplitkPlan splitk_plan(int64_t M, int64_t N, int64_t K, bool gu, bool allow_spli
         best.cnt_bytes + (size_t)best.S * best.nb * sk::part_floats(best.mt, best.tw, gu, best.x1, best.nw) * 4;
   }
   return best;
+}
+
+// The model runs over up to 96 candidates, twice per call (selection and
+// launch): a thread keeps its last plans, one per slot of a small table, a
+// pure function of the key.
+SplitkPlan splitk_plan(int64_t M, int64_t N, int64_t K, bool gu, bool allow_split) {
+  const int cus = device_cus();
+#ifndef RA_TUNING
+  struct Entry {
+    int64_t M = -1, N, K;
+    int flags, cus;
+    SplitkPlan p;
+  };
+  constexpr int kSlots = 64;
+  thread_local Entry table[kSlots];
+  const int flags = (gu ? 2 : 0) | (allow_split ? 1 : 0);
+  Entry &e = table[((uint64_t)M * 31 + (uint64_t)N * 7 + (uint64_t)K * 13 + (uint64_t)flags * 3) / 8 % kSlots];
+  if (e.M != M || e.N != N || e.K != K || e.flags != flags || e.cus != cus)
+    e = Entry{M, N, K, flags, cus, make_plan(M, N, K, gu, allow_split, cus)};
+  return e.p;
+#else
+  return make_plan(M, N, K, gu, allow_split, cus);
+#endif
 }
 
 namespace {

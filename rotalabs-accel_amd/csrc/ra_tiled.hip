@@ -823,8 +823,6 @@ static bool tiled_split_eligible(const GemmArgs &a) {
          tiled_supported(a) && dma_span_ok(false, a.ldx, a.ldw, a.N, a.K, (int)std::max<int64_t>(a.M, 256));
 }
 
-static int device_cus();
-
 // Split-K plans for the small tile (M = 33..64): 64-row tiles of 64*bnb
 // weight rows (2 x 2 waves of bnb 32x32 blocks), K split over nsplit
 // workgroups per tile. Time model fitted to the same-run times of every
@@ -1026,14 +1024,6 @@ static int small_grid_rows(int64_t M, int64_t N, bool gu, int cus) {
 static int64_t large_tile_count(int64_t M, int64_t N, int cus) {
   const DmaShape c = pick_dma_shape(M, N, false, cus);
   return ((M + c.bm() - 1) / c.bm()) * ((N + c.bn() - 1) / c.bn());
-}
-
-static int device_cus() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    return 256;
-  return cus;
 }
 
 template <int DT, bool GU>

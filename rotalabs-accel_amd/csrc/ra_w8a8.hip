@@ -482,14 +482,6 @@ static void launch_tiles(const W8A8Args &a, hipStream_t s) {
     }
 }
 
-static int device_cus() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    return 256;
-  return cus;
-}
-
 template <int DT, int I = 0>
 static void launch_cfg(int idx, const W8A8Args &a, hipStream_t s) {
   if constexpr (I < kNumCfgs) {

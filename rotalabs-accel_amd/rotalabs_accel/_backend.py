@@ -10,12 +10,15 @@ Set ``ROTACCEL_LIB`` to load the library from another path.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
 import torch
 
 _LIB_DEFAULT = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "librotaccel.so")
+_HOST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "_ra_host.so")
 _lock = threading.Lock()
 _lib = None
 _load_error: str | None = None
@@ -48,6 +51,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "ra_w8a16_gemm_ex": ([p, i64, i32, p, i64, p, p, i32, p, i64, i64, i64, i64, i32, p, sz, p], i32),
         "ra_w8a16_gemm_ws": ([p, i64, i32, p, i64, p, p, i32, p, i64, i64, i64, i64, p, sz, p], i32),
         "ra_w8a16_gemm_workspace_size": ([i64, i64, i64, i32], sz),
+        "ra_w8a16_gemm_auto_workspace": ([i64, i64, i64, i32], sz),
         "ra_w8a16_gemm_noalloc": ([p, i64, i32, p, i64, p, p, i32, p, i64, i64, i64, i64, p], i32),
         "ra_w8a16_gateup_swiglu_ws": ([p, i64, i32, p, i64, p, p, i64, i64, i64, i64, p, sz, p], i32),
         "ra_w8a16_gateup_workspace_size": ([i64, i64, i64, i32], sz),
@@ -68,6 +72,26 @@ def _declare(lib: ctypes.CDLL) -> None:
         fn = getattr(lib, name)
         fn.argtypes = args
         fn.restype = res
+
+
+def _load_host():
+    """The native host path (csrc/host/ra_host.cpp), or None where it is not
+    built: the ops then take the Python path to the same library."""
+    if not os.path.exists(_HOST_PATH):
+        return None
+    loader = importlib.machinery.ExtensionFileLoader("_ra_host", _HOST_PATH)
+    spec = importlib.util.spec_from_file_location("_ra_host", _HOST_PATH, loader=loader)
+    try:
+        module = importlib.util.module_from_spec(spec)
+        loader.exec_module(module)
+    except ImportError:
+        return None
+    return module
+
+
+# Its functions return None until load() has succeeded, and for every call that
+# is not the plain case.
+host = _load_host()
 
 
 def load():
@@ -91,6 +115,8 @@ def load():
         ver = lib.ra_abi_version()
         if ver != ABI_VERSION:
             raise RuntimeError(f"rotalabs_accel: {path} has ABI {ver}, expected {ABI_VERSION}; rebuild it")
+        if host is not None:
+            host.init(path, _workspaces, _host_workspace)
         _lib = lib
         return lib
 
@@ -192,6 +218,10 @@ def workspace(device: torch.device, nbytes: int):
             _held.append(ws)
     assert ws.data_ptr() % WORKSPACE_ALIGN == 0
     return ws.data_ptr(), ws.numel()
+
+
+def _host_workspace(device_index: int, nbytes: int):
+    return workspace(torch.device("cuda", device_index), nbytes)
 
 
 class on_device:

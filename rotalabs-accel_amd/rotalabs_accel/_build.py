@@ -33,6 +33,7 @@ INCLUDE = os.path.join(REPO_DIR, "include")
 BUILD_DIR = os.path.join(PROJ_DIR, "_build")
 LIB_DIR = os.path.join(PKG_DIR, "_lib")
 LIB_PATH = os.path.join(LIB_DIR, "librotaccel.so")
+HOST_PATH = os.path.join(LIB_DIR, "_ra_host.so")
 
 ARCH = "gfx950"
 
@@ -69,8 +70,32 @@ def _compile_one(src: str) -> str:
     return obj
 
 
+def build_host() -> str:
+    """Compile csrc/host/ra_host.cpp (host code only) against the installed
+    torch's headers into _lib/_ra_host.so. Returns its path."""
+    import sysconfig
+
+    import torch
+    troot = os.path.dirname(os.path.abspath(torch.__file__))
+    lib = os.path.join(troot, "lib")
+    cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-shared",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{troot}/include", f"-I{troot}/include/torch/csrc/api/include",
+           f"-I{os.path.join(os.environ.get('ROCM_PATH', '/opt/rocm'), 'include')}", f"-I{INCLUDE}",
+           f"-I{sysconfig.get_paths()['include']}", os.path.join(CSRC, "host", "ra_host.cpp"),
+           "-o", HOST_PATH + ".tmp", f"-L{lib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python",
+           f"-Wl,-rpath,{lib}"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"host extension failed:\n{res.stderr}")
+    os.replace(HOST_PATH + ".tmp", HOST_PATH)
+    return HOST_PATH
+
+
 def build(verbose: bool = False) -> str:
-    """Compile every csrc/*.hip for gfx950 and link librotaccel.so. Returns its path."""
+    """Compile every csrc/*.hip for gfx950 and link librotaccel.so, then the
+    host extension. Returns the library's path."""
     os.makedirs(BUILD_DIR, exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
     sources = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
@@ -85,6 +110,7 @@ def build(verbose: bool = False) -> str:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
+    build_host()
     if verbose:
         print(f"built {LIB_PATH} from {len(sources)} sources")
     return LIB_PATH

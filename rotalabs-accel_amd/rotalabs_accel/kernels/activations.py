@@ -12,6 +12,7 @@ import torch
 import torch.nn.functional as F
 
 from rotalabs_accel import _backend
+from rotalabs_accel._backend import host as _host
 
 
 def swiglu_torch(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
@@ -20,6 +21,10 @@ def swiglu_torch(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
 
 def swiglu_fused(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     """``silu(gate) * up`` elementwise."""
+    if _host is not None:
+        out = _host.swiglu(gate, up)
+        if out is not None:
+            return out
     assert gate.shape == up.shape, f"Shape mismatch: gate={gate.shape}, up={up.shape}"
     if gate.is_cuda and up.is_cuda:
         lib = _backend.load()

@@ -26,6 +26,7 @@ import torch
 import torch.nn.functional as F
 
 from rotalabs_accel import _backend
+from rotalabs_accel._backend import host as _host
 from rotalabs_accel.quantization.symmetric import dequantize, quantize_weight_per_channel
 
 
@@ -150,6 +151,10 @@ def int8_gemm(
     Returns:
         (..., N) tensor of x's dtype.
     """
+    if _host is not None:
+        y = _host.gemm(x, weight_int8, scale, bias)
+        if y is not None:
+            return y
     assert weight_int8.dtype == torch.int8, "Weight must be INT8"
     K = x.shape[-1]
     N = weight_int8.shape[0]

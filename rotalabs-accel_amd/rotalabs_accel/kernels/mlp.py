@@ -24,6 +24,7 @@ from typing import Optional
 import torch
 
 from rotalabs_accel import _backend
+from rotalabs_accel._backend import host as _host
 from rotalabs_accel.kernels.activations import SwiGLU, swiglu_fused, swiglu_torch
 from rotalabs_accel.kernels.gemm import _rows, _workspace_size, int8_gemm, int8_gemm_torch
 from rotalabs_accel.kernels.normalization import rmsnorm, rmsnorm_residual_fused
@@ -36,6 +37,10 @@ def int8_gateup_swiglu(x: torch.Tensor, weight_gate_up: torch.Tensor, scale_gate
     x: (..., K); weight_gate_up: int8 (2I, K); scale_gate_up: fp32 (2I,).
     Returns (..., I) in x's dtype.
     """
+    if _host is not None:
+        h = _host.gateup(x, weight_gate_up, scale_gate_up)
+        if h is not None:
+            return h
     assert weight_gate_up.dtype == torch.int8, "Weight must be INT8"
     K = x.shape[-1]
     n2 = weight_gate_up.shape[0]
@@ -69,6 +74,10 @@ def int8_mlp(x: torch.Tensor, norm_weight: torch.Tensor, weight_gate_up: torch.T
              eps: float = 1e-6, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
     """RMSNorm (of ``x + residual`` when given) -> fused gate/up + SwiGLU ->
     down projection."""
+    if _host is not None:
+        y = _host.mlp(x, residual, norm_weight, eps, weight_gate_up, scale_gate_up, weight_down, scale_down)
+        if y is not None:
+            return y
     if residual is not None:
         h = rmsnorm_residual_fused(x, residual, norm_weight, eps)
     else:

@@ -14,6 +14,7 @@ from __future__ import annotations
 import torch
 
 from rotalabs_accel import _backend
+from rotalabs_accel._backend import host as _host
 
 
 def rmsnorm_torch(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:
@@ -83,6 +84,10 @@ def _rmsnorm_residual_hip(x: torch.Tensor, residual: torch.Tensor, weight: torch
 
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:
     """RMS normalisation over the last dimension, times ``weight``."""
+    if _host is not None:
+        y = _host.rmsnorm(x, None, weight, eps)
+        if y is not None:
+            return y
     assert x.shape[-1] == weight.shape[0], f"Hidden dim mismatch: {x.shape[-1]} vs {weight.shape[0]}"
     if x.is_cuda and weight.is_cuda:
         return _rmsnorm_hip(x, weight, eps)
@@ -92,6 +97,10 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.T
 def rmsnorm_residual_fused(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
                            eps: float = 1e-6) -> torch.Tensor:
     """RMSNorm of ``x + residual`` times ``weight`` (one pass on the GPU)."""
+    if _host is not None and residual is not None:
+        y = _host.rmsnorm(x, residual, weight, eps)
+        if y is not None:
+            return y
     assert x.shape == residual.shape, f"Shape mismatch: x={x.shape}, residual={residual.shape}"
     assert x.shape[-1] == weight.shape[0], f"Hidden dim mismatch: {x.shape[-1]} vs {weight.shape[0]}"
     if x.is_cuda and residual.is_cuda and weight.is_cuda:

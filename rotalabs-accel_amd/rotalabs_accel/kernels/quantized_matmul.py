@@ -35,6 +35,7 @@ from typing import Optional
 import torch
 
 from rotalabs_accel import _backend
+from rotalabs_accel._backend import host as _host
 from rotalabs_accel.kernels import gemm as _gemm
 from rotalabs_accel.kernels.gemm import Int8Linear, int8_gemm_torch  # noqa: F401  (re-exported as there)
 
@@ -174,6 +175,10 @@ def int8_gemm(
     assert scale.shape == (N,), f"Scale shape mismatch: {scale.shape} vs ({N},)"
     x2 = x.reshape(-1, K)
     if use_cublas and x2.shape[0] >= W8A8_MIN_M:
+        if _host is not None:
+            y = _host.w8a8(x, weight_int8, scale, bias, ACT_SCALE)
+            if y is not None:
+                return y
         x_int8, x_scale = quantize_activations(x2)
         y = w8a8_gemm(x_int8, x_scale, weight_int8, scale, bias)
         return y.view(*x.shape[:-1], N)

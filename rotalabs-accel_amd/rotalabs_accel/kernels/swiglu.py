@@ -20,6 +20,7 @@ import torch
 import torch.nn.functional as F
 
 from rotalabs_accel import _backend
+from rotalabs_accel._backend import host as _host
 from rotalabs_accel.kernels.activations import swiglu_fused, swiglu_torch
 
 __all__ = ["swiglu_fused", "swiglu_torch", "SwiGLU", "swiglu_with_bias"]
@@ -46,6 +47,10 @@ def swiglu_with_bias(
 ) -> torch.Tensor:
     """``silu(gate + bias_gate) * (up + bias_up)``; biases of shape (hidden,)
     broadcast over the last dimension of gate / up. Output dtype = gate's."""
+    if _host is not None:
+        out = _host.swiglu_bias(gate, up, bias_gate, bias_up)
+        if out is not None:
+            return out
     assert gate.shape == up.shape
     assert gate.shape[-1] == bias_gate.shape[0] == bias_up.shape[0]
     if not gate.is_cuda:

@@ -20,6 +20,7 @@ from typing import Optional
 import torch
 
 from rotalabs_accel import _backend
+from rotalabs_accel._backend import host as _host
 
 _QMAX = 127
 
@@ -53,6 +54,10 @@ def quantize_symmetric(
 
 def _quantize_rows_hip(w: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     lib = _backend.load()
+    if _host is not None:
+        qs = _host.quantize(w)
+        if qs is not None:
+            return qs
     if w.stride(-1) != 1:
         w = w.contiguous()
     n, k = w.shape

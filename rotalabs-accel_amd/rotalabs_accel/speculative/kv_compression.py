@@ -15,6 +15,7 @@ from __future__ import annotations
 import torch
 
 from rotalabs_accel import _backend
+from rotalabs_accel._backend import host as _host
 
 _KERNEL_DTYPES = (torch.float16, torch.bfloat16, torch.float32)
 
@@ -47,6 +48,10 @@ class QuantizedTensor:
     @staticmethod
     def _quantize_rows_hip(tensor: torch.Tensor, bits: int):
         lib = _backend.load()
+        if _host is not None:
+            qs = _host.kv_quantize(tensor, bits)
+            if qs is not None:
+                return qs
         cols = tensor.shape[-1]
         t2 = tensor.reshape(-1, cols)
         if t2.stride(-1) != 1 or (t2.shape[0] > 1 and t2.stride(0) < cols):
@@ -63,6 +68,10 @@ class QuantizedTensor:
 
     def dequantize(self) -> torch.Tensor:
         q, s = self.data, self.scale
+        if _host is not None and isinstance(s, torch.Tensor) and s.dtype == self.dtype:
+            out = _host.kv_dequantize(q, s)
+            if out is not None:
+                return out
         if isinstance(s, torch.Tensor) and q.is_cuda and q.dtype == torch.int8 and s.device == q.device \
                 and s.dtype == self.dtype and s.dtype in _KERNEL_DTYPES and q.dim() > 0 \
                 and s.shape == q.shape[:-1] + (1,) and q.is_contiguous() and s.is_contiguous() \
