@@ -135,6 +135,10 @@ __global__ __launch_bounds__(64 * NWT, 1) void splitk_kernel(const char *__restr
   constexpr int XS = x_slot(MT), WS = w_slot(TW, GU);
   constexpr int XRING = 0, WRING = (D + 1) * XS, X1RING = WRING + D * NWT * WS;
   constexpr int R = NWT * TW * 16;  // output columns per unit
+  // K % 128 != 0 (a last stage that overlaps the one before): the GEMM without
+  // the extra row (whose kernels slow by 3 % with it: M=17 K=28672 N=8192
+  // 42.4 against 43.4 us)
+  constexpr bool TAIL = !GU && X1 == 0;
   constexpr int X1L = 16 / NWT;     // lanes per wave copying the extra row (16 bytes each)
   static_assert(X1 == 0 || X1 == 1, "at most one row past the MFMA tiles");
   static_assert(NWT == 4 || NWT == 8, "4 or 8 waves per workgroup");
@@ -161,7 +165,7 @@ __global__ __launch_bounds__(64 * NWT, 1) void splitk_kernel(const char *__restr
   const int n0 = rb * R;
   const int kb = s * kc;
   const int ke = min(K, kb + kc);
-  const int nst = (ke - kb + KS - 1) / KS;  // >= 1 (host)
+  const int nst = (ke - kb + (TAIL ? KS - 1 : 0)) / KS;  // >= 1 (host)
   // Row block rb walks its stages starting at stage rb % nst (wrapping), so
   // the units in flight read different k windows. In lockstep they would all
   // read the same window, addresses equal in their low log2(ldw) bits, which
@@ -213,7 +217,7 @@ __global__ __launch_bounds__(64 * NWT, 1) void splitk_kernel(const char *__restr
 
   auto issue = [&](int st) __attribute__((always_inline)) {
     const int sr = st + rot < nst ? st + rot : st + rot - nst;
-    const int k = min(kb + sr * KS, K - KS);  // K % 128 != 0: the last stage ends at K
+    const int k = TAIL ? min(kb + sr * KS, K - KS) : kb + sr * KS;  // K % 128 != 0: the last stage ends at K
     const char *sw = wb + k;
     const char *sx = xb + (int64_t)k * 2;
     const uint32_t wd = wdst + (uint32_t)((st % D) * NWT * WS);
@@ -259,7 +263,7 @@ __global__ __launch_bounds__(64 * NWT, 1) void splitk_kernel(const char *__restr
     // every fragment read cost the other stages up to 6 %). Same run, bf16,
     // us, against the kernels that took such K before: N=4096 K=11040 M=4
     // 17.1 -> 15.6, M=16 20.3 -> 16.7, M=64 47.6 -> 26.4.
-    if constexpr (!GU) {
+    if constexpr (TAIL) {
       const int skip = kb + (st + rot < nst ? st + rot : st + rot - nst) * KS + KS - K;
       if (skip > 0) {  // uniform over the workgroup
         const int nc = skip / 8;
@@ -268,9 +272,6 @@ __global__ __launch_bounds__(64 * NWT, 1) void splitk_kernel(const char *__restr
           const int row = i / nc, c = i - row * nc;
           store16(xz + row * 256 + ((c ^ (row & 15)) << 4), make_uint4(0, 0, 0, 0));
         }
-        if constexpr (X1 != 0)
-          if ((int)threadIdx.x < nc)
-            store16(lds + X1RING + (st % (D + 1)) * x1_slot + 16 * threadIdx.x, make_uint4(0, 0, 0, 0));
         __syncthreads();
       }
     }
@@ -512,7 +513,7 @@ static SplitkPlan make_plan(int64_t M, int64_t N, int64_t K, bool gu, bool allow
   best.ok = false;
   if (M < 1 || M > sk::kMaxM || K < sk::KS || K % (gu ? sk::KS : 32) != 0 || N < 1) return best;
   int mt = sk_mt(M), x1 = 0;
-  if (x1_wanted(M, K, gu)) {
+  if (K % sk::KS == 0 && x1_wanted(M, K, gu)) {
     mt = (int)(M / 16);
     x1 = 1;
   }
