@@ -451,15 +451,24 @@ __global__ __launch_bounds__(256, OCC_) void w8a8_gemm_kernel(const int8_t *__re
 // stages, OCC workgroups per CU. `cost` is the relative time per output
 // when every CU is busy (measured at prefill shapes, M = 512..8192). Two
 // workgroups per CU (to overlap one's epilogue with the other's loop) and
-// 64-k stages measured slower; the 64-k configuration serves K % 128 == 64.
+// 64-k stages measured slower there; 64-k stages serve K % 128 == 64.
+// The first kNumSmall are for small grids, the first whose tiles fit one
+// round of the CUs: a tile's time is nearly its K loop's (64 x 64 about 0.18
+// us per 128 k, 64 x 128 0.27, 128 x 128 0.30, 128 x 192 0.39, 256 x 128 0.49
+// before the CUs fill up), so the smallest that leaves no second round wins.
+// fp16, us, 256-row tiles -> these: K=11008 N=4096 M=17 49.6 -> 19.4, M=512
+// 56.4 -> 34.2; K=4096 N=4096 M=200 25.9 -> 12.6, M=1024 29.2 -> 24.4;
+// K=4096 N=11008 M=100 28.2 -> 16.4, M=512 30.7 -> 29.0 (128 x 192). K=1024
+// N=16384 M=350 (none fits) keeps 17.8.
 struct Cfg {
   int bmb, bnb, bk, occ;
   double cost;
 };
 constexpr Cfg kCfgs[] = {
-    {4, 4, 128, 1, 1.00}, {4, 3, 128, 1, 1.05}, {4, 2, 128, 1, 1.10}, {4, 2, 64, 1, 1.10},
+    {1, 1, 128, 2, 0.0},  {1, 2, 128, 2, 0.0},  {2, 2, 128, 1, 0.0},  {2, 3, 128, 1, 0.0},  {1, 2, 64, 2, 0.0},
+    {2, 2, 64, 2, 0.0},   {4, 4, 128, 1, 1.00}, {4, 3, 128, 1, 1.05}, {4, 2, 128, 1, 1.10}, {4, 2, 64, 1, 1.10},
 };
-constexpr int kNumCfgs = sizeof(kCfgs) / sizeof(kCfgs[0]);
+constexpr int kNumCfgs = sizeof(kCfgs) / sizeof(kCfgs[0]), kNumSmall = 6;
 
 template <int DT, int BMB, int BNB, int BK, int OCC>
 static void launch_tiles(const W8A8Args &a, hipStream_t s) {
@@ -491,8 +500,9 @@ static void launch_cfg(int idx, const W8A8Args &a, hipStream_t s) {
   }
 }
 
-// Tiles run in rounds of (CUs x workgroups per CU); the configuration with
-// the least (rounds x tile area x relative cost) wins.
+// A small-grid configuration that fits, else tiles run in rounds of the CUs
+// and the configuration with the least (rounds x tile area x relative cost)
+// wins.
 template <int DT>
 static void launch_dt(const W8A8Args &a, hipStream_t s) {
   const int cus = device_cus();
@@ -501,9 +511,14 @@ static void launch_dt(const W8A8Args &a, hipStream_t s) {
   for (int i = 0; i < kNumCfgs; ++i) {
     const Cfg &c = kCfgs[i];
     if (a.K % c.bk != 0 || (c.bk == 64 && a.K % 128 == 0)) continue;
-    const int64_t bm = 64 * c.bmb, bn = 64 * c.bnb, slots = (int64_t)cus * c.occ;
+    const int64_t bm = 64 * c.bmb, bn = 64 * c.bnb;
     const int64_t tiles = ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
-    const double t = (double)((tiles + slots - 1) / slots) * (double)(bm * bn) * c.cost / c.occ;
+    if (i < kNumSmall) {
+      if (tiles > cus) continue;
+      pick = i;
+      break;
+    }
+    const double t = (double)((tiles + cus - 1) / cus) * (double)(bm * bn) * c.cost;
     if (pick < 0 || t < best_t) pick = i, best_t = t;
   }
 #ifdef RA_TUNING
