@@ -235,6 +235,16 @@ int ra_swiglu(const void *gate, const void *up, void *out, int64_t n,
               int dtype, void *stream);
 
 /*
+ * ra_swiglu of the two halves of gate_up [rows, 2 * hidden] (row stride ld >=
+ * 2 * hidden elements, gate columns first) into out [rows, hidden]
+ * (contiguous): the activation between a biased gate/up projection and the
+ * down projection (SwiGLU.forward, src/rotalabs_accel/kernels/
+ * activations.py:165-178).
+ */
+int ra_swiglu_halves(const void *gate_up, int64_t ld, void *out,
+                     int64_t rows, int64_t hidden, int dtype, void *stream);
+
+/*
  * out = silu(gate + bias_gate[i % hidden]) * (up + bias_up[i % hidden]) over
  * n = rows * hidden contiguous elements (dtype), biases [hidden] in
  * bias_dtype; fp32 math, one rounding. Replaces swiglu_with_bias

@@ -549,6 +549,15 @@ int ra_swiglu(const void *gate, const void *up, void *out, int64_t n, int dtype,
   return to_status(swiglu_launch(gate, up, out, n, dtype, static_cast<hipStream_t>(stream)));
 }
 
+int ra_swiglu_halves(const void *gate_up, int64_t ld, void *out, int64_t rows, int64_t hidden, int dtype,
+                     void *stream) {
+  if (rows < 0 || hidden < 0 || rows > INT32_MAX || hidden > INT32_MAX) return RA_ERR_ARG;
+  if (!valid_act(dtype)) return RA_ERR_DTYPE;
+  if (rows == 0 || hidden == 0) return RA_OK;
+  if (!gate_up || !out || ld < 2 * hidden) return RA_ERR_ARG;
+  return to_status(swiglu_halves_launch(gate_up, ld, out, rows, hidden, dtype, static_cast<hipStream_t>(stream)));
+}
+
 int ra_swiglu_bias(const void *gate, const void *up, const void *bias_gate, const void *bias_up, int bias_dtype,
                    void *out, int64_t n, int64_t hidden, int dtype, void *stream) {
   if (n < 0 || hidden <= 0 || n % hidden != 0) return RA_ERR_ARG;

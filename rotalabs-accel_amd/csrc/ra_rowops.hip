@@ -202,7 +202,8 @@ hipError_t rmsnorm_launch(const void *x, int64_t ldx, int x_dt, const void *r, i
 
 // out = silu(g) * u = g / (1 + exp(-g)) * u in fp32, one rounding
 // (the Triton kernel's arithmetic, src/rotalabs_accel/kernels/activations.py:69-80).
-__device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
+// (fp32_rounded: the product is rounded to fp32, then to 16 bits, in every form.)
+__device__ __forceinline__ float silu_mul(float g, float u) { return fp32_rounded(g / (1.0f + expf(-g)) * u); }
 
 // Bound by HBM (two values read, one written per element). One 16-byte chunk
 // of gate and of up per lane: 2-byte accesses moved a quarter of what the
@@ -263,6 +264,50 @@ static hipError_t swiglu_any(const void *g, const void *u, const void *bg, const
     hipLaunchKernelGGL((swiglu_kernel<RA_BF16, BIAS>), grid, block, 0, s, g, u, bg, bu, b_dt, o, n, hidden);
   else
     hipLaunchKernelGGL((swiglu_kernel<RA_F32, BIAS>), grid, block, 0, s, g, u, bg, bu, b_dt, o, n, hidden);
+  return hipGetLastError();
+}
+
+// The same over the two halves of [rows, 2 * hidden] (a gate/up product with
+// its biases added, gate columns first): the halves are read in place, where
+// two copies made them contiguous before (M=2048 I=11008 bf16: 22.1 after 2 x 16.2 us of copies -> 23.2).
+// INROW: hidden is a whole number of chunks, so a chunk stays in its row.
+template <int DT, bool INROW>
+__global__ __launch_bounds__(256) void swiglu_halves_kernel(const void *__restrict__ gu, int64_t ld,
+                                                            void *__restrict__ o, int64_t n, int64_t hidden) {
+  using C = Chunk<DT>;
+  const int64_t step = (int64_t)gridDim.x * 256 * C::E;
+  for (int64_t i0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * C::E; i0 < n; i0 += step) {
+    int64_t row = n <= INT32_MAX ? (int64_t)((uint32_t)i0 / (uint32_t)hidden) : i0 / hidden;
+    int64_t col = i0 - row * hidden;
+    if constexpr (INROW) {
+      const char *gp = static_cast<const char *>(gu) + (row * ld + col) * C::SZ;
+      const uint4 gc = load16_any(gp), uc = load16_any(gp + hidden * C::SZ);
+      uint4 oc;
+#pragma unroll
+      for (int e = 0; e < C::E; ++e) C::set(oc, e, silu_mul(C::get(gc, e), C::get(uc, e)));
+      store16_any(static_cast<char *>(o) + i0 * C::SZ, oc);
+    } else {
+      for (int64_t i = i0; i < i0 + C::E && i < n; ++i) {
+        store_from_f32(o, i, DT, silu_mul(load_as_f32(gu, row * ld + col, DT), load_as_f32(gu, row * ld + hidden + col, DT)));
+        if (++col == hidden) col = 0, ++row;
+      }
+    }
+  }
+}
+
+hipError_t swiglu_halves_launch(const void *gu, int64_t ld, void *o, int64_t rows, int64_t hidden, int dt,
+                                hipStream_t s) {
+  const int64_t n = rows * hidden, per = 256 * (dt == RA_F32 ? 4 : 8);
+  const dim3 grid((unsigned)std::min((n + per - 1) / per, kSwigluMaxBlocks)), block(256);
+#define RA_HALVES(DT_)                                                                                     \
+  if (dt == DT_) {                                                                                         \
+    if (hidden % Chunk<DT_>::E == 0)                                                                       \
+      hipLaunchKernelGGL((swiglu_halves_kernel<DT_, true>), grid, block, 0, s, gu, ld, o, n, hidden);      \
+    else                                                                                                   \
+      hipLaunchKernelGGL((swiglu_halves_kernel<DT_, false>), grid, block, 0, s, gu, ld, o, n, hidden);     \
+  }
+  RA_HALVES(RA_F16) RA_HALVES(RA_BF16) RA_HALVES(RA_F32)
+#undef RA_HALVES
   return hipGetLastError();
 }
 

@@ -69,6 +69,22 @@ def int8_gateup_swiglu(x: torch.Tensor, weight_gate_up: torch.Tensor, scale_gate
     return h.view(*x.shape[:-1], inter)
 
 
+def _swiglu_halves(gu: torch.Tensor) -> torch.Tensor:
+    """``swiglu_fused`` of the two halves of ``gu`` (..., 2I), read in place on
+    the GPU."""
+    inter = gu.shape[-1] // 2
+    if not gu.is_cuda or not gu.is_contiguous():
+        return swiglu_fused(gu[..., :inter].contiguous(), gu[..., inter:].contiguous())
+    lib = _backend.load()
+    out = torch.empty((*gu.shape[:-1], inter), dtype=gu.dtype, device=gu.device)
+    if out.numel() == 0:
+        return out
+    with _backend.on_device(gu.device):
+        _backend.check(lib.ra_swiglu_halves(gu.data_ptr(), 2 * inter, out.data_ptr(), out.numel() // inter, inter,
+                                            _backend.dtype_code(gu.dtype), _backend.stream_handle(gu.device)))
+    return out
+
+
 def int8_mlp(x: torch.Tensor, norm_weight: torch.Tensor, weight_gate_up: torch.Tensor,
              scale_gate_up: torch.Tensor, weight_down: torch.Tensor, scale_down: torch.Tensor,
              eps: float = 1e-6, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -167,7 +183,7 @@ class Int8SwiGLU(torch.nn.Module):
     ``bias_gate_up`` [2I] and ``bias_down`` [H] (fp16 like ``Int8Linear``'s).
     Without biases the gate and up projections run as one GEMM with SwiGLU in
     its epilogue (``int8_gateup_swiglu``); with biases they run as one biased
-    GEMM, then ``swiglu_fused``. CPU tensors run the same composition with the
+    GEMM, then the activation of its two halves. CPU tensors run the same composition with the
     PyTorch ops.
     """
 
@@ -226,7 +242,7 @@ class Int8SwiGLU(torch.nn.Module):
             a = int8_gateup_swiglu(x, self.weight_gate_up, self.scale_gate_up)
         else:
             gu = int8_gemm(x, self.weight_gate_up, self.scale_gate_up, self.bias_gate_up)
-            a = swiglu_fused(gu[..., :inter].contiguous(), gu[..., inter:].contiguous())
+            a = _swiglu_halves(gu)
         return int8_gemm(a, self.weight_down, self.scale_down, self.bias_down)
 
     def extra_repr(self) -> str:

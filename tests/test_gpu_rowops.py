@@ -109,3 +109,16 @@ def test_rmsnorm_odd_rows(gpu, dt, wide, rows, hidden):
         n = fallback.rmsnorm_exact_ref(v.float().numpy(), one, 1e-6, name)
         ref = (torch.from_numpy(n) * w.float()).to(w.dtype)
         assert y.dtype == w.dtype and torch.equal(y, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", HALF + [torch.float32])
+@pytest.mark.parametrize("rows,hidden", [(1, 1), (3, 5), (7, 8), (5, 333), (6, 4104), (300, 2049), (0, 16)])
+def test_swiglu_halves_same_bits(gpu, dt, rows, hidden):
+    """The halves read in place give what their contiguous copies give."""
+    from rotalabs_accel.kernels.mlp import _swiglu_halves
+    g = torch.Generator().manual_seed(hidden)
+    gu = (torch.randn(rows, 2 * hidden, generator=g) * 3).to(dt).to(gpu)
+    print(f"  swiglu halves {dt} [{rows}, {hidden}]", flush=True)
+    ref = ra.swiglu_fused(gu[:, :hidden].contiguous(), gu[:, hidden:].contiguous())
+    assert torch.equal(_swiglu_halves(gu), ref)
