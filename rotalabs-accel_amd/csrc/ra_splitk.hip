@@ -117,7 +117,7 @@ __device__ __forceinline__ void wait_stages(int younger) {
 // row is a dot product on the VALU (v_dot2 over the weights the MFMA tiles
 // already dequantised), instead of a second, almost empty 16-row MFMA tile
 // (whose activation copies, LDS reads and MFMAs cost as much as a full one).
-template <int DT, int MT, int TW, bool GU, int X1, int DMAX = sk::kMaxD, int NWT = sk::NW>
+template <int DT, int MT, int TW, bool GU, int X1, int DMAX = sk::kMaxD, int NWT = sk::NW, bool TAIL = false>
 __global__ __launch_bounds__(64 * NWT, 1) void splitk_kernel(const char *__restrict__ xb, int64_t ldx,
                                                         const char *__restrict__ wb, int64_t ldw,
                                                         const float *__restrict__ scale,
@@ -135,10 +135,9 @@ __global__ __launch_bounds__(64 * NWT, 1) void splitk_kernel(const char *__restr
   constexpr int XS = x_slot(MT), WS = w_slot(TW, GU);
   constexpr int XRING = 0, WRING = (D + 1) * XS, X1RING = WRING + D * NWT * WS;
   constexpr int R = NWT * TW * 16;  // output columns per unit
-  // K % 128 != 0 (a last stage that overlaps the one before): the GEMM without
-  // the extra row (whose kernels slow by 3 % with it: M=17 K=28672 N=8192
-  // 42.4 against 43.4 us)
-  constexpr bool TAIL = !GU && X1 == 0;
+  // TAIL: K % 128 != 0, a last stage that overlaps the one before. Kernels of
+  // their own (it slowed the others by up to 3 %), without an extra row.
+  static_assert(!TAIL || (!GU && X1 == 0), "no tail stage here");
   constexpr int X1L = 16 / NWT;     // lanes per wave copying the extra row (16 bytes each)
   static_assert(X1 == 0 || X1 == 1, "at most one row past the MFMA tiles");
   static_assert(NWT == 4 || NWT == 8, "4 or 8 waves per workgroup");
@@ -610,9 +609,11 @@ void splitk_go(const SplitkPlan &p, const void *x, int64_t ldx, const int8_t *w,
   const unsigned grid = (unsigned)(p.spread ? (int64_t)p.nb * p.S : ((p.nb + 7) / 8) * 8 * p.S);
   int *cnt = static_cast<int *>(ws);
   float *part = ws ? reinterpret_cast<float *>(static_cast<char *>(ws) + p.cnt_bytes) : nullptr;
-  if (NWT != sk::NW) {  // 8 waves per workgroup
-    hipLaunchKernelGGL((splitk_kernel<DT, MT, TW, GU, X1, sk::kMaxD, NWT>), dim3(grid), dim3(64 * NWT), 0, s,
-                       static_cast<const char *>(x), ldx, reinterpret_cast<const char *>(w), ldw, scale, bias,
+  constexpr bool TAILS = !GU && X1 == 0;  // (other plans come with whole stages)
+  if (NWT != sk::NW || (TAILS && K % sk::KS != 0)) {  // 8 waves per workgroup, or a tail stage
+    auto *const kernel = TAILS && K % sk::KS != 0 ? splitk_kernel<DT, MT, TW, GU, X1, sk::kMaxD, NWT, TAILS>
+                                                  : splitk_kernel<DT, MT, TW, GU, X1, sk::kMaxD, NWT>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * NWT), 0, s, static_cast<const char *>(x), ldx, reinterpret_cast<const char *>(w), ldw, scale, bias,
                        bias_dt, static_cast<uint16_t *>(y), ldy, (int)M, (int)N, (int)K, p.kc, p.S, p.nb,
                        p.spread ? 1 : 0, part, cnt);
     return;

@@ -245,9 +245,10 @@ __global__ __launch_bounds__(256, 2) void tiled_kernel(const uint16_t *__restric
 // K % 64 != 0, pad k's short of whole tiles: tile 1 starts at 64 - pad, and so
 // on to a last tile that ends at K (no copy leaves the rows, and only tile 0
 // is off the common origin); the activations in tile 0 of the k's that tile 1
-// holds too are cleared in LDS before the first read, so the K loop is the
-// same code. (Moving the last tile instead, or masking fragments, slowed the
-// whole multiples: M=2048 K=4096 N=8192 103 -> 126 us.) The register-staged
+// holds too are cleared in LDS before the first read (TAIL, kernels of their
+// own: the prologue's few instructions more cost the 64 x 64 tile 1.8 % at
+// M=64 K=4096 N=11008, and moving the last tile instead, or masking
+// fragments, M=2048 K=4096 N=8192 103 -> 126 us). The register-staged
 // kernel above ran these with 256-row tiles, whatever M, and no split (bf16,
 // us, N=4096 K=11040: M=100 224 -> 33, M=2048 247 -> 157).
 // ---------------------------------------------------------------------------
@@ -318,7 +319,7 @@ __device__ __forceinline__ int uniform_if(int v) {
 constexpr int kMaxTileSplits = 4;  // K splits per tile of the SPLIT form
 constexpr int kMaxTileBmb = 2;     // 32x32 row blocks per wave of the SPLIT form (tiles of 64 or 128 rows)
 
-template <int DT, bool GU, int BMB, int BNB, int WR, int SM = 4, bool SPLIT = false>
+template <int DT, bool GU, int BMB, int BNB, int WR, int SM = 4, bool SPLIT = false, bool TAIL = false>
 __global__ __launch_bounds__(256, (DmaTile<BMB, BNB, WR, SM>::PER_CU)) void tiled_dma_kernel(const uint16_t *__restrict__ x, int64_t ldx,
                                                            const int8_t *__restrict__ w, int64_t ldw,
                                                            const float *__restrict__ scale,
@@ -403,8 +404,8 @@ __global__ __launch_bounds__(256, (DmaTile<BMB, BNB, WR, SM>::PER_CU)) void tile
     }
     b_voff[i] = (uint32_t)((int64_t)wr * ldw + c * 16) + (uint32_t)(DMA_BIAS - (i % 4) * 1024);
   }
-  const int KTA = (K + BK - 1) / BK;  // K tiles in all
-  const int pad = KTA * BK - K;       // k's that tiles 0 and 1 share
+  const int KTA = TAIL ? (K + BK - 1) / BK : K / BK;  // K tiles in all
+  const int pad = TAIL ? KTA * BK - K : 0;            // k's that tiles 0 and 1 share
   const char *const xb = reinterpret_cast<const char *>(x) - DMA_BIAS - 2 * pad;
   const char *const wb = reinterpret_cast<const char *>(w) - DMA_BIAS - pad;
   const uint32_t lds0 = lds_offset(lds);
@@ -558,15 +559,17 @@ constexpr int P1 = (COPIES + 2) / 3, P2 = (2 * COPIES + 2) / 3;
   __builtin_amdgcn_sched_barrier(0);
 
   const int KT = SPLIT ? min(KTA - kt0, ksplit) : KTA;  // K tiles of this workgroup (>= 1)
-  const bool short0 = pad > 0 && kt0 == 0;              // this workgroup's tile 0 overlaps tile 1
-  const int ko0 = uniform_if<SPLIT && (BMB > 1)>(short0 ? pad : kt0 * BK);
-  RA_ISSUE_AT(ko0, 0, 0, COPIES);
+  const bool short0 = TAIL && kt0 == 0;                 // this workgroup's tile 0 overlaps tile 1
+  if constexpr (TAIL) {
+    const int ko0 = uniform_if<SPLIT && (BMB > 1)>(short0 ? pad : kt0 * BK);
+    RA_ISSUE_AT(ko0, 0, 0, COPIES);
+  }
 #pragma unroll
-  for (int s = 1; s < S; ++s)
+  for (int s = TAIL ? 1 : 0; s < S; ++s)
     if (s < KT) RA_ISSUE(s, s);
   wait_tiles<COPIES, S - 1>(min(KT, S) - 1);
   asm volatile("s_barrier" ::: "memory");
-  if (short0) {
+  if (TAIL && short0) {
     const int c0 = (BK - pad) / 8, nc = 8 - c0;
     for (int i = tid; i < BM * nc; i += 256) {
       const int row = i / nc, c = c0 + i - row * nc;
@@ -933,8 +936,9 @@ static void launch_dma_split(const GemmArgs &a, const TiledSplitPlan &p, void *w
   const int tiles_m = (int)((a.M + G::BM - 1) / G::BM);
   int *cnt = static_cast<int *>(ws);
   float *part = p.nsplit > 1 ? reinterpret_cast<float *>(static_cast<char *>(ws) + kSplitkCounterBytes) : nullptr;
-  hipLaunchKernelGGL((tiled_dma_kernel<DT, false, BMB, BNB, 2, 6, true>), dim3((unsigned)(tiles_m * tiles_n * p.nsplit)),
-                     dim3(256), 0, s, static_cast<const uint16_t *>(a.x), a.ldx, a.w, a.ldw, a.scale, a.bias,
+  auto *const kernel = a.K % G::BK ? tiled_dma_kernel<DT, false, BMB, BNB, 2, 6, true, true>
+                                   : tiled_dma_kernel<DT, false, BMB, BNB, 2, 6, true, false>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles_m * tiles_n * p.nsplit)), dim3(256), 0, s, static_cast<const uint16_t *>(a.x), a.ldx, a.w, a.ldw, a.scale, a.bias,
                      a.bias_dt, static_cast<uint16_t *>(a.y), a.ldy, (int)a.M, (int)a.N, (int)a.K, tiles_m, tiles_n,
                      p.nsplit, p.ksplit, part, cnt);
 }
@@ -967,7 +971,9 @@ static void launch_dma(const void *x, int64_t ldx, const int8_t *w, int64_t ldw,
 #else
       float *trace = nullptr;
 #endif
-      hipLaunchKernelGGL((tiled_dma_kernel<DT, GU, BMB, BNB, WR, SM>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, s,
+      auto *const kernel = K % G::BK ? tiled_dma_kernel<DT, GU, BMB, BNB, WR, SM, false, true>
+                                     : tiled_dma_kernel<DT, GU, BMB, BNB, WR, SM, false, false>;
+      hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, s,
                          xi, ldx, w + ns * ldw, ldw, si, bi, bias_dt, yi, ldy, (int)Mi, (int)Ni, (int)K, tiles_m,
                          tiles_n, 1, 0, trace, nullptr);
     }
