@@ -239,7 +239,7 @@ int ra_swiglu(const void *gate, const void *up, void *out, int64_t n,
  * 2 * hidden elements, gate columns first) into out [rows, hidden]
  * (contiguous): the activation between a biased gate/up projection and the
  * down projection (SwiGLU.forward, src/rotalabs_accel/kernels/
- * activations.py:165-178).
+ * activations.py:141-181).
  */
 int ra_swiglu_halves(const void *gate_up, int64_t ld, void *out,
                      int64_t rows, int64_t hidden, int dtype, void *stream);
@@ -285,7 +285,7 @@ int ra_quantize_rows(const void *t, int64_t ldt, int t_dtype,
 
 /*
  * The codec's way back (QuantizedTensor.dequantize, src/rotalabs_accel/
- * speculative/kv_compression.py:80-84): out[r,c] = q[r,c] * scale[r] in fp32,
+ * speculative/kv_compression.py:51-88): out[r,c] = q[r,c] * scale[r] in fp32,
  * rounded once to t_dtype. q: int8 [rows, cols]; scale: [rows] and out:
  * [rows, cols] in t_dtype, all contiguous.
  */
