@@ -645,6 +645,10 @@ constexpr int P1 = (COPIES + 2) / 3, P2 = (2 * COPIES + 2) / 3;
       constexpr int CH = BMB * BNB * 4;  // 16-byte chunks per lane
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
           part + (size_t)t * nsplit * 4 * CH * 256, 0, nsplit * 4 * CH * 256 * (int)sizeof(float), kRsrcWord3);
+      // Row groups past M are neither exchanged nor stored (M=200 K=11008
+      // N=4096: 22 % of the partial sums, 44.2 -> 42.2 us).
+      const int row_g = m0 + wm * WM + 4 * g;
+      auto live = [&](int bi, int q) { return row_g + 32 * bi + 8 * q < M; };
       auto off = [&](int split, int c) { return (uint32_t)((((split * 4 + wid) * CH + c) * 64 + lane) * 16); };
 #pragma unroll
       for (int bi = 0; bi < BMB; ++bi)
@@ -653,7 +657,7 @@ constexpr int P1 = (COPIES + 2) / 3, P2 = (2 * COPIES + 2) / 3;
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             const f32x16 &a = acc[bi][bj];
-            store_dev16(rs, off(sp, (bi * BNB + bj) * 4 + q), f32x4{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]});
+            if (live(bi, q)) store_dev16(rs, off(sp, (bi * BNB + bj) * 4 + q), f32x4{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]});
           }
       wait_vmcnt<0>();  // this wave's partial sums are stored
       __syncthreads();  // and every wave's
@@ -674,7 +678,8 @@ constexpr int P1 = (COPIES + 2) / 3, P2 = (2 * COPIES + 2) / 3;
         for (int s2 = 0; s2 < kMaxTileSplits; ++s2)
 #pragma unroll
           for (int c = 0; c < CG; ++c)
-            if (g0 + c < NC && s2 < nsplit && s2 != sp) o[s2][c] = load_dev16(rs, off(s2, g0 + c));
+            if (g0 + c < NC && s2 < nsplit && s2 != sp && live((g0 + c) / (BNB * 4), (g0 + c) % 4))
+              o[s2][c] = load_dev16(rs, off(s2, g0 + c));
 #pragma unroll
         for (int c = 0; c < CG; ++c) {
           if (g0 + c >= NC) break;
